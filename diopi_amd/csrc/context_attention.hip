@@ -1077,8 +1077,8 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnPipe(T* 
 // ---- heads of 64 ----
 //
 // Half the products of a head of 128 come with each score, and the softmax keeps its precision: the probabilities take part in
-// the second product as the sum of two 16-bit numbers (16 significant bits in bf16, 21 in fp16), whose row sums are taken in fp32
-// before the split.  So of the 64 x 32 scores of a wave and tile it is the vector work that bounds the kernel (a fused multiply-add,
+// the second product as the sum of two 16-bit numbers (see SplitPair: 17 significant bits in bf16, 23 in fp16), whose row sums are
+// taken in fp32 before the split.  So of the 64 x 32 scores of a wave and tile it is the vector work that bounds the kernel (a fused multiply-add,
 // an exponential of 4 issue slots, half a maximum, a sum, 2-3 instructions of splitting for each score), with 8 + 16 products
 // beside it.  Against the pipelined kernel above the balance is the other way round: what pays is more waves a SIMD, which
 // fill each other's waits without a hand-made schedule, so the registers are kept to 3 waves a SIMD: no
@@ -1090,23 +1090,30 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnPipe(T* 
 // slots of a 256-byte line, and the swizzle is by the row pair:
 //   K tile: slot s of row r holds packet s ^ ((r / 2) & 7)        (16 lanes reading one packet of 16 rows hit 16 slots)
 //   V tile: slot s of row r holds packet s ^ (4 * ((r / 2) & 1))  (the 4 packets of 4 rows that a transposing read takes, too)
+// Both halves are rounded to nearest, so what a split leaves off has no direction.  Where a new reference puts a row's largest
+// probability, and how large one may grow before the reference moves again (powers of two): fp16 runs out of exponents at 2^-24,
+// so its probabilities are kept as large as they can be, 2^11 .. 2^15 for the largest, and what is left off is at most 2^-36 of that one
+// (with the largest at 1 and halves cut toward zero 32768 keys 2^-20 below one other came out 2.5 % short; now within 2^-16).
 template <typename T>
 struct SplitPair;
 template <>
 struct SplitPair<half_t> {
+    static constexpr float kTopLog2 = 11.f, kMostLog2 = 15.f;
     static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& lo) {
-        const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        const h2 h = __builtin_convertvector((f32x2{a, b}), h2);
         hi = __builtin_bit_cast(uint32_t, h);
-        lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a - static_cast<float>(h[0]), b - static_cast<float>(h[1])));
+        lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a - static_cast<float>(h[0]), b - static_cast<float>(h[1])}), h2));
     }
 };
 template <>
 struct SplitPair<bf16_t> {
+    static constexpr float kTopLog2 = 0.f, kMostLog2 = kLazyLog2;
     static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& lo) {
         typedef float f32x2 __attribute__((ext_vector_type(2)));
-        const uint32_t ab = __builtin_bit_cast(uint32_t, a), bb = __builtin_bit_cast(uint32_t, b);
-        hi = __builtin_amdgcn_perm(bb, ab, 0x07060302u);  // the upper halves: truncated, what is left is exact
-        const f32x2 rest = {a - __builtin_bit_cast(float, ab & 0xffff0000u), b - __builtin_bit_cast(float, bb & 0xffff0000u)};
+        hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+        const f32x2 rest = {a - __builtin_bit_cast(float, hi << 16), b - __builtin_bit_cast(float, hi & 0xffff0000u)};
         lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, bf16x2));
     }
 };
@@ -1300,10 +1307,11 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 3 : 2) void ctxAttn64(T* __
         }
         const float tmA = max3(tm[0], s[0][7], s[0][15]), tmB = max3(tm[1], s[1][7], s[1][15]);
         const float tmax = maxWithOtherHalf(max3(max3(tmA, tmB, tm[2]), tm[3], tm[3]));
-        // the reference follows the true maximum only when it lags by more than 2^kLazyLog2 (see ctxAttnMfma)
+        // the reference follows the true maximum only when a probability would come out above 2^kMostLog2 (see SplitPair)
+        using Split = SplitPair<T>;
         const float lag = __builtin_fmaf(tmax, scaleLog2, negRef);
-        if (jt == 0 || __any(lag > kLazyLog2)) {
-            const float up = jt == 0 ? lag : fmaxf(lag, 0.f);
+        if (jt == 0 || __any(lag > Split::kMostLog2)) {
+            const float up = jt == 0 ? lag - Split::kTopLog2 : fmaxf(lag - Split::kTopLog2, 0.f);
             const float alpha = __builtin_amdgcn_exp2f(-up);
             negRef -= up;
             if (jt > 0) {
@@ -1327,7 +1335,7 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 3 : 2) void ctxAttn64(T* __
                 none[2 * w] = p0 == 0.f;
                 none[2 * w + 1] = p1 == 0.f;
                 uint32_t hw, lw;
-                SplitPair<T>::split(p0, p1, hw, lw);
+                Split::split(p0, p1, hw, lw);
                 h.raw[w] = hw;
                 l.raw[w] = lw;
             }
@@ -1427,8 +1435,11 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 3 : 2) void ctxAttn64(T* __
     // ---- normalise, transpose through LDS, write rows with 16-byte stores ----
     const float lTot = lRun + __shfl_xor(lRun, 32, kWave);
     const float inv = 1.0f / lTot;
-    if (a.lse != nullptr && hh == 0 && qRow < L && qRow < a.lseStride)
-        a.lse[(static_cast<int64_t>(planned.x) * a.H + head) * a.lseStride + qRow] = 0.6931471805599453f * (__builtin_amdgcn_logf(lTot) - negRef);
+    if (a.lse != nullptr && hh == 0 && qRow < L && qRow < a.lseStride) {
+        constexpr float kTop = SplitPair<T>::kTopLog2;  // taken out of both terms: neither is larger, or rounds coarser, for it
+        a.lse[(static_cast<int64_t>(planned.x) * a.H + head) * a.lseStride + qRow] =
+            0.6931471805599453f * (__builtin_amdgcn_logf(lTot * __builtin_amdgcn_exp2f(-kTop)) + (kTop - negRef));
+    }
     waitLdsLoads();
     __syncthreads();  // the tiles are dead and no request is in flight
     T* sO = smem;

@@ -142,6 +142,30 @@ def test_attention(dt, causal, H, Hkv, scale):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,gap", [(16384, 10), (16384, 14), (32768, 20)])
+def test_attention_one_key_over_many(dt, n, gap):
+    """A key far above all others, whose own value is zero: what comes out is the sum of many small probabilities."""
+    g = torch.Generator().manual_seed(gap)
+    q, k, v = torch.zeros(n, 1, 64), torch.zeros(n, 1, 64), torch.rand(n, 1, 64, generator=g) + 0.5
+    q[:, 0, 0] = 8
+    k[:, 0, 0] = torch.randn(n, generator=g).clamp(-3, 3) * np.log(2)
+    k[5, 0, 0] = gap * np.log(2)
+    v[:, 0, :32] = 1
+    v[5] = 0
+    q, k, v = (t.to(dt).to(DEV) for t in (q, k, v))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    out = F.flash_attention_varlen(q, k, v, cu, cu, None, n, n, 0.0, None, False)[:, 0].double()
+    p = k[:, 0, 0].double().softmax(0)  # q . k / 8
+    want = p @ v[:, 0].double()
+    u, tiny = ROUND[dt]
+    # the exponent of a score of at most 16 powers of two, scaled, shifted and taken in fp32; a rounding for each half of 16 keys, within
+    # and after a tile; the halves of a probability (2^-17, and in fp16 2^-36 of the largest); the result's rounding
+    rel = 64 * 2.0 ** -24 + (n / 8 + 64) * 2.0 ** -24 + 2.0 ** -17
+    bound = rel * want + (n * 2.0 ** -36 * p.max() * 1.5 if dt == torch.float16 else 0.0) + u * want + tiny
+    assert ((out - want).abs() <= 1.01 * bound).all(), float(((out - want) / want).abs().max())
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_attention_values_that_are_no_numbers(dt):
     """What a row does not see leaves it alone: infinities and NaN among later rows' values, wherever the row stands in its tile."""
     lens = [200, 64, 33]
