@@ -1613,8 +1613,9 @@ diopiError_t dispatchAttention(diopiContextHandle_t ctx, hipStream_t stream, con
     const bool planFits = (4 * static_cast<int64_t>(a.batch) + a.rows / kBMMin + 1) * 4 <= 64 * 1024 && a.rows <= INT32_MAX;
     // the tile requests address a 64-row tile with 32-bit byte offsets
     const bool tileFits = static_cast<int64_t>(a.H) * kHD * 8 * kBN < INT32_MAX;
-    // the kernel for heads of 64 takes the largest score for the largest after scaling
-    const bool scales = softmaxScale > 0.0 && softmaxScale < 1e30;
+    // the kernel for heads of 64 takes the largest score for the largest after scaling, and a masked score of -inf for -inf: a scale that
+    // fp32 holds as zero would make a NaN of it
+    const bool scales = softmaxScale > 1e-30 && softmaxScale < 1e30;
     const bool fast = (D == kHD || (D == 64 && scales)) && aligned && planFits && tileFits;
     // 256-row query tiles (8 waves share each K/V tile) once the sequences are long enough to fill them
     const bool wide = a.rows >= 1024 * static_cast<int64_t>(a.batch);

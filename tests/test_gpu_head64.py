@@ -194,6 +194,16 @@ def test_attention_odd_scales(scale):
     assert ((out - general).abs() <= 3 * 2.0 ** -11 * general.abs() + 1e-3).all()
 
 
+def test_attention_scale_that_fp32_holds_as_zero():
+    """All keys weigh the same, and masked ones nothing."""
+    q, k, v, _ = _packed([130], 2, 2, torch.float16, 8)
+    q, k, v = (t.view(1, 130, 2, 64) for t in (q, k, v))
+    out, general = (F.multihead_attention(q, k, t, 0.0, True, False, 1e-50) for t in (v, _unaligned(v)))
+    want = v.double().cumsum(1) / torch.arange(1, 131, device=DEV, dtype=torch.float64).view(1, -1, 1, 1)
+    assert ((out.double() - want).abs() <= 2.0 ** -11 * want.abs() + 130 * 2.0 ** -23 * 4 + 2.0 ** -25).all()
+    assert ((out - general).abs() <= 2 * 2.0 ** -11 * general.abs() + 1e-4).all()
+
+
 def test_attention_where_no_plan_can_be_had():
     """The allocation-free entry point with more query tiles than its static plan holds: refused for heads of 128, for heads of 64
     the general kernel takes the call, as it did every one."""
