@@ -303,13 +303,19 @@ diopiError_t launchStaged(hipStream_t stream, void* out, const void* q, const vo
     // sequences of 512..2048 tokens, 32 heads); with 8 query heads per kv head (128 sequences of 1024..8192 tokens, 8 kv
     // heads) 256 is 4 % faster than 128 and 512 is 1 % slower than 256: longer pieces of every logits row per write-out
     int TT = a.G == 1 ? 64 : 256;
+    // A launch has 65535 tiles at most, so a window (max_input_len) that long takes tiles as long as every call once had: shorter ones
+    // are no reason to refuse it.
+    const int longest = HD == 64 ? 128 : TT;
+    int shortest = 64;
+    while (shortest < longest && ceilDiv(a.maxInputLen, shortest) > 65535) shortest *= 2;
+    if (TT < shortest) TT = shortest;
     const int gridX = static_cast<int>(ceilDiv(pieces, HS * HW));
     // Shorter tiles where those leave compute units idle, until there are two work-groups for each (256 and 64 tokens: one
     // sequence of 4000 tokens with 8 kv heads of 4 query heads 16.4 and 6.6 us, 8 of 500..2000 with the same heads 18.3 and 7.6,
     // 24 of 128..3001 with heads of 64 22.6 and 12.8; 2 of 20001 and 50001 with 8 of 8, 555 work-groups of 256 tokens: 36.3 and 39.4)
     const int64_t wantedGroups = 2 * static_cast<int64_t>(deviceInfo().numCU);
     const int64_t tokens = tokensAtMost(a);
-    while (TT > 64 && gridX * ceilDiv(tokens, TT) < wantedGroups) TT /= 2;
+    while (TT > shortest && gridX * ceilDiv(tokens, TT) < wantedGroups) TT /= 2;
     const bool fewGroups = gridX * ceilDiv(tokens, TT) < wantedGroups;
     // the scores of a tile wait in LDS for the write-out: at most 40 KiB of them
     const int outRows = HS * HW * HP * a.G;

@@ -95,6 +95,36 @@ def test_token_attention(dt, H, Hkv, idt):
         assert ((got[0] - want).abs() <= 1.01 * bound)[fine].all() and ((got[0] - got[1]).abs() <= 2.02 * bound)[fine].all(), (i, n)
 
 
+def _in_window(w, window):
+    table = torch.zeros(w["B"], window, dtype=torch.int32, device=DEV)
+    table[:, -w["longest"]:] = w["b_loc"]
+    return table, w["b_start"], w["b_len"], window
+
+
+@pytest.mark.parametrize("H,Hkv,window", [(2, 2, 65535 * 64 + 1), (4, 1, 65535 * 128)])
+def test_token_attention_long_windows(H, Hkv, window):
+    """Windows of more tiles of 64 tokens than a launch can have: only their last columns are in use."""
+    w = _decode([70, 200], H, Hkv, torch.float16, torch.int32, 31)
+    out, short = (torch.zeros(H, w["total"], dtype=torch.float16, device=DEV) for _ in range(2))
+    F.token_attention(w["q"], w["k"], out, *_in_window(w, window))
+    F.token_attention(w["q"], w["k"], short, w["b_loc"], w["b_start"], w["b_len"], w["longest"])
+    assert torch.equal(out, short)
+
+
+def test_token_attention_long_window_of_grouped_heads():
+    """Heads of 128 in groups had tiles of 256 tokens whatever the number of cached tokens."""
+    H, Hkv, D, window, n = 8, 2, 128, 65535 * 64 + 1, 100
+    g = torch.Generator().manual_seed(32)
+    q, k = (torch.randn(s, generator=g).half().to(DEV) for s in ((1, H, D), (n, Hkv, D)))
+    table = torch.zeros(1, window, dtype=torch.int32, device=DEV)
+    table[0, -n:] = torch.arange(n)
+    start, length = (torch.tensor([x], dtype=torch.int32, device=DEV) for x in (0, n))
+    out, short = (torch.zeros(H, n, dtype=torch.float16, device=DEV) for _ in range(2))
+    F.token_attention(q, k, out, table, start, length, window)
+    F.token_attention(q, k, short, table[:, -n:].contiguous(), start, length, n)
+    assert torch.equal(out, short)
+
+
 def _packed(lens, H, Hkv, dt, seed):
     g = torch.Generator().manual_seed(seed)
     q, k, v = (torch.randn(sum(lens), h, 64, generator=g).to(dt).to(DEV) for h in (H, Hkv, Hkv))
