@@ -30,6 +30,7 @@ constexpr int kRvWaves = kRvThreads / kWave;
 constexpr int kSub = 128;          // tokens per sub-tile
 constexpr int kD = 128;            // dims of a cache row that a work-group takes: one head of 128 or two of 64
 constexpr int kMaxGroup = 16;      // query heads of a work-group: rows of a matrix instruction
+constexpr int kShortest = kRvWaves * kSub;  // shortest range of a work-group for heads of 64: a sub-tile for each of four waves
 
 struct SplitArgs {
     float* partAcc;  // [batch, splits, H, D]
@@ -552,7 +553,6 @@ diopiError_t launchWave(diopiContextHandle_t ctx, hipStream_t stream, void* out,
         // two heads to a work-group make fewer of them: shorter ranges until there are two for each compute unit, a sub-tile for
         // every wave at least, no sequence of up to 1024 tokens cut (24 sequences of 128..3001 tokens with 8 kv heads of 4 query
         // heads, whole as 96 work-groups of 16 waves 24.6 us, in ranges of 512 tokens 16.8)
-        constexpr int kShortest = kRvWaves * kSub;
         while (TT > kShortest && a.maxInputLen > 2 * kShortest && groups() < 2 * numCU) TT = TT / 2 > kShortest ? static_cast<int>(ceilDiv(TT / 2, kSub)) * kSub : kShortest;
     }
     sp.TT = TT;
@@ -643,7 +643,8 @@ diopiError_t tokenSoftmaxReduceV(diopiContextHandle_t ctx, const TensorView& vOu
     ROCM_CALL(getStream(ctx, &stream));
     // the matrix-core kernel keeps slot numbers in 32 bits, reads V rows with 16-byte loads and addresses the G logits
     // rows of a kv head with a 32-bit byte offset
-    const bool mfma = (a.D == 128 || a.D == 64) && a.G <= kMaxGroup && a.numSlots < (int64_t(1) << 31) && (reinterpret_cast<uintptr_t>(vV.data) & 15) == 0 &&
+    // and heads of 64 leave windows (max_input_len) of more ranges than a launch takes to the general kernel, which has no such limit
+    const bool mfma = (a.D == 128 || (a.D == 64 && a.maxInputLen <= 65535 * kShortest)) && a.G <= kMaxGroup && a.numSlots < (int64_t(1) << 31) && (reinterpret_cast<uintptr_t>(vV.data) & 15) == 0 &&
                       a.logitCols * 16 * 2 < (int64_t(1) << 31);
     switch (vOut.dtype) {
         case diopi_dtype_float16:

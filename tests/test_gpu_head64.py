@@ -125,6 +125,15 @@ def test_token_attention_long_window_of_grouped_heads():
     assert torch.equal(out, short)
 
 
+def test_softmax_reducev_long_window():
+    """A window of more ranges of 512 tokens than a launch can have."""
+    w = _decode([70, 200], 2, 1, torch.float16, torch.int32, 31)
+    out, general = (torch.zeros(2, 2, 64, dtype=torch.float16, device=DEV) for _ in range(2))
+    F.token_softmax_reducev(w["logits"], w["v"], out, *_in_window(w, 65535 * 512 + 1), 0)
+    F.token_softmax_reducev(w["logits"], _unaligned(w["v"]), general, w["b_loc"], w["b_start"], w["b_len"], w["longest"], 0)
+    assert torch.equal(out, general)
+
+
 def _packed(lens, H, Hkv, dt, seed):
     g = torch.Generator().manual_seed(seed)
     q, k, v = (torch.randn(sum(lens), h, 64, generator=g).to(dt).to(DEV) for h in (H, Hkv, Hkv))
