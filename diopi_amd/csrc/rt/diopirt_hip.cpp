@@ -81,7 +81,7 @@ constexpr int64_t kBlockAlign = 1024;  // the reference stub rounds every alloca
 
 int64_t roundUp(int64_t n, int64_t a) { return (n + a - 1) / a * a; }
 
-void* poolTake(PooledContext* ctx, int64_t bytes, diopiDevice_t device, int64_t* capacity) {
+void* poolTake(PooledContext* ctx, int64_t bytes, diopiDevice_t device, bool mayAllocate, int64_t* capacity) {
     auto& freeList = device == diopi_device ? ctx->freeDevice : ctx->freeHost;
     int64_t want = roundUp(bytes > 0 ? bytes : 1, kBlockAlign);
     auto it = freeList.lower_bound(want);
@@ -92,6 +92,7 @@ void* poolTake(PooledContext* ctx, int64_t bytes, diopiDevice_t device, int64_t*
         freeList.erase(it);
         return p;
     }
+    if (!mayAllocate) return nullptr;
     void* p = nullptr;
     if (device == diopi_device) {
         if (hipMalloc(&p, want) != hipSuccess) return nullptr;
@@ -103,9 +104,20 @@ void* poolTake(PooledContext* ctx, int64_t bytes, diopiDevice_t device, int64_t*
     return p;
 }
 
+// Allocating while the stream is captured would end the capture: a request that the pool cannot serve is refused then.
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 diopiTensor* PooledContext::keepScratch(diopiTensor* t, int64_t bytes) {
+    const bool mayAllocate = t->device != diopi_device || !capturing(getStream());
     std::lock_guard<std::mutex> lock(mtx);
-    t->data = poolTake(this, bytes, t->device, &t->capacity);
+    t->data = poolTake(this, bytes, t->device, mayAllocate, &t->capacity);
     if (!t->data) return nullptr;
     inUse += t->capacity;
     if (inUse > peak) peak = inUse;
