@@ -161,13 +161,16 @@ diopiError_t getStream(diopiContextHandle_t ctx, hipStream_t* stream) {
 diopiError_t requireScratch(diopiContextHandle_t ctx, int64_t bytes, void** ptr) {
     ROCM_CHECK(ctx != nullptr, "the context handle is null");
     diopiTensorHandle_t t = nullptr;
-    if (diopiRequireBuffer != nullptr) {
-        ROCM_CHECK(diopiRequireBuffer(ctx, &t, bytes, diopi_device) == diopiSuccess && t != nullptr, "diopiRequireBuffer(%lld bytes) failed",
-                   static_cast<long long>(bytes));
-    } else {
-        diopiSize_t size{&bytes, 1};
-        ROCM_CHECK(diopiRequireTensor(ctx, &t, &size, nullptr, diopi_dtype_int8, diopi_device) == diopiSuccess && t != nullptr,
-                   "diopiRequireTensor(%lld bytes) failed", static_cast<long long>(bytes));
+    const bool buffer = diopiRequireBuffer != nullptr;
+    diopiSize_t size{&bytes, 1};
+    const diopiError_t err = buffer ? diopiRequireBuffer(ctx, &t, bytes, diopi_device)
+                                    : diopiRequireTensor(ctx, &t, &size, nullptr, diopi_dtype_int8, diopi_device);
+    if (err != diopiSuccess || t == nullptr) {
+        // what the caller's allocator left behind is its own: the next launch check must not find it
+        const hipError_t left = hipGetLastError();
+        if (left != hipSuccess) noteHipError(left);
+        setLastErrorAt(__FILE__, __LINE__, "%s(%lld bytes) failed", buffer ? "diopiRequireBuffer" : "diopiRequireTensor", static_cast<long long>(bytes));
+        return diopiErrorOccurred;
     }
     ROCM_CHECK(diopiGetTensorData(t, ptr) == diopiSuccess && *ptr != nullptr, "scratch tensor has no data pointer");
     return diopiSuccess;

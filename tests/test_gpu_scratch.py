@@ -76,3 +76,19 @@ def test_a_refused_call_leaves_a_capture_valid():
     torch.cuda.synchronize()
     assert_close(out[0, 0], v[0, 0], rtol=2.0 ** -10, atol=2.0 ** -24, what="the same call outside")
     ctx.close()
+
+
+def test_memory_that_the_device_does_not_have():
+    """The call that asked for it fails; the next one is not held responsible."""
+    ctx = rt.Context()
+    window, H = 65535 * 2048, 16384  # 558 GB of partial sums
+    v = torch.randn(4, H, 128).half().to(DEV)
+    logits, out = torch.zeros(H, 4, dtype=torch.float16, device=DEV), torch.zeros(1, H, 128, dtype=torch.float16, device=DEV)
+    table, start, length = torch.zeros(1, window, dtype=torch.int32, device=DEV), *(torch.tensor([x], dtype=torch.int32, device=DEV) for x in (0, 4))
+    for c in (ctx, None):
+        with pytest.raises(rt.DiopiException, match="failed"):
+            F.token_softmax_reducev(logits, v, out, table, start, length, window, 0, ctx=c)
+        F.token_softmax_reducev(logits, v, out, table, start, length, 2048, 0, ctx=c)
+        torch.cuda.synchronize()
+        assert_close(out[0], v[0], rtol=2.0 ** -10, atol=2.0 ** -24, what="the next call")
+    ctx.close()
