@@ -74,7 +74,7 @@ struct PooledContext : diopiContext {
     diopiTensor* keepScratch(diopiTensor* tensor, int64_t bytes) override;
 };
 
-// Every handle that diopirtContextCreate made is one of these; the diopirtContext* calls take no others.
+// Every handle that diopirtContextCreate or diopirtContextAdopt made is one of these; the diopirtContext* calls take no others.
 PooledContext* pooled(diopiContextHandle_t ctx) { return static_cast<PooledContext*>(ctx); }
 
 constexpr int64_t kBlockAlign = 1024;  // the reference stub rounds every allocation to 1 KiB (litert.hpp:57-59)
@@ -156,14 +156,14 @@ int diopirtDeviceComputeUnits(int device) {
     return n;
 }
 
-diopiContextHandle_t diopirtContextCreate(void* stream) {
+diopiContextHandle_t diopirtContextAdopt(void* stream) {
     auto* ctx = new PooledContext();
-    if (stream != nullptr) {
-        ctx->stream = static_cast<hipStream_t>(stream);
-        ctx->adopted = true;
-    }
+    ctx->stream = static_cast<hipStream_t>(stream);
+    ctx->adopted = true;
     return ctx;
 }
+
+diopiContextHandle_t diopirtContextCreate(void* stream) { return stream != nullptr ? diopirtContextAdopt(stream) : new PooledContext(); }
 
 void diopirtContextClearTensors(diopiContextHandle_t handle) {
     PooledContext* ctx = pooled(handle);
@@ -182,7 +182,7 @@ void diopirtContextClearTensors(diopiContextHandle_t handle) {
 void diopirtContextDestroy(diopiContextHandle_t handle) {
     PooledContext* ctx = pooled(handle);
     if (!ctx) return;
-    if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->stream || ctx->adopted) (void)hipStreamSynchronize(ctx->stream);
     diopirtContextClearTensors(ctx);
     for (auto& kv : ctx->freeDevice) (void)hipFree(kv.second);
     for (auto& kv : ctx->freeHost) std::free(kv.second);

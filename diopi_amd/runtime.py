@@ -116,6 +116,8 @@ class _Libs:
         rt.diopirtDeviceComputeUnits.restype, rt.diopirtDeviceComputeUnits.argtypes = i32, [i32]
         rt.diopirtContextCreate.restype = vp
         rt.diopirtContextCreate.argtypes = [vp]
+        if hasattr(rt, "diopirtContextAdopt"):  # an older build pointed to has none: its contexts adopt no null stream
+            rt.diopirtContextAdopt.restype, rt.diopirtContextAdopt.argtypes = vp, [vp]
         rt.diopirtContextDestroy.argtypes = [vp]
         rt.diopirtContextClearTensors.argtypes = [vp]
         rt.diopirtContextSynchronize.argtypes = [vp]
@@ -261,7 +263,9 @@ class Context:
         if stream is None and not own_stream and torch.cuda.is_available():
             self.torch_stream = torch.cuda.Stream()
         handle = self.torch_stream.cuda_stream if self.torch_stream is not None else None
-        self.handle = ctypes.c_void_p(self._rt.diopirtContextCreate(ctypes.c_void_p(handle)))
+        # the handle of torch's default stream is zero, which asks diopirtContextCreate for a stream of the context's own
+        create = self._rt.diopirtContextAdopt if handle == 0 else self._rt.diopirtContextCreate
+        self.handle = ctypes.c_void_p(create(ctypes.c_void_p(handle)))
 
     def synchronize(self) -> None:
         ret = self._rt.diopirtContextSynchronize(self.handle)

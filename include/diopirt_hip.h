@@ -36,6 +36,8 @@ int diopirtDeviceComputeUnits(int device);
 /* Create a context.  `stream` is an existing hipStream_t to adopt, or NULL to
  * let the context create its own non-blocking stream on first use. */
 diopiContextHandle_t diopirtContextCreate(void* stream);
+/* Create a context on an existing hipStream_t, NULL being the null stream. */
+diopiContextHandle_t diopirtContextAdopt(void* stream);
 /* Destroys the context, its own stream (if it created one) and its scratch pool. */
 void diopirtContextDestroy(diopiContextHandle_t ctx);
 /* Hands every tensor given out by diopiRequireTensor/Buffer back to the pool.

@@ -94,3 +94,21 @@ def test_calls_without_a_context_in_a_hip_graph():
         want = _step(*args)
         for a, b, name in zip(got, want, ("grad_input", "grad_weight", "logits", "decode out")):
             assert_bit_equal(a, b, f"replay {replay}: {name}")
+
+
+@pytest.mark.gpu
+def test_context_on_torchs_default_stream():
+    """Its handle is null: the operator still runs behind what torch has queued there, and torch behind the operator."""
+    ctx = rt.Context(stream=torch.cuda.default_stream())
+    a = torch.randn(4096, 4096, device=DEV)
+    cache, dest = torch.zeros(4, 1, 64, device=DEV), torch.tensor([1], dtype=torch.int32, device=DEV)
+    row = torch.zeros(1, 1, 64, device=DEV)
+    torch.cuda.synchronize()
+    for n in range(1, 6):
+        for _ in range(20):  # some milliseconds of work in front of the row that the operator reads
+            a = a @ a * 1e-2
+        row.copy_((a[:1, :64] * 0 + n).view(1, 1, 64))
+        F.destindex_copy_kv(row, dest, cache, ctx=ctx)
+        seen = cache.clone()
+        assert float(seen[1, 0, 0]) == n and float(seen[1, 0, 63]) == n
+    ctx.close()
