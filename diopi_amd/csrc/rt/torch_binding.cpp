@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
+#include <atomic>
 #include <tuple>
 #include <utility>
 
@@ -47,6 +48,9 @@ bool dtypeOf(c10::ScalarType s, diopiDtype_t* dtype) {
     }
 }
 
+// Scratch of the calls on torch's current stream, all threads together, in blocks as a context's pool counts them.
+std::atomic<int64_t> scratchInUse{0}, scratchPeak{0};
+
 // The context of one call on torch's current stream.  Its scratch goes back to torch's allocator when the call has
 // queued its work; a later owner on this stream is ordered behind it.
 struct CurrentStreamContext final : diopiContext {
@@ -55,6 +59,7 @@ struct CurrentStreamContext final : diopiContext {
         c10::DataPtr memory;
     };
     std::vector<Scratch> scratch;
+    int64_t held = 0;
 
     hipStream_t getStream() override { return c10::hip::getCurrentHIPStream().stream(); }
 
@@ -65,6 +70,11 @@ struct CurrentStreamContext final : diopiContext {
             t->data = memory.get();
             if (t->data == nullptr) return nullptr;
             scratch.push_back({t, std::move(memory)});
+            const int64_t block = (bytes > 0 ? bytes + 1023 : 1024) / 1024 * 1024;
+            held += block;
+            const int64_t now = scratchInUse.fetch_add(block) + block;
+            for (int64_t peak = scratchPeak.load(); peak < now && !scratchPeak.compare_exchange_weak(peak, now);) {
+            }
             return t;
         } catch (const std::exception&) {
             return nullptr;  // out of memory: the operator reports that its scratch was refused
@@ -73,6 +83,7 @@ struct CurrentStreamContext final : diopiContext {
 
     ~CurrentStreamContext() override {
         for (auto& s : scratch) delete s.tensor;
+        scratchInUse.fetch_sub(held);
     }
 };
 
@@ -239,6 +250,8 @@ struct Operator<Fn> {
     }
 };
 
+PyObject* scratchPeakOf(PyObject*, PyObject*) { return PyLong_FromLongLong(scratchPeak.load()); }
+
 #define DIOPI_BOUND(name) \
     { #name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Operator<&name>::entry)), METH_FASTCALL, nullptr }
 PyMethodDef kMethods[] = {
@@ -262,6 +275,7 @@ PyMethodDef kMethods[] = {
     DIOPI_BOUND(diopiRootMeanSquareNormInp),
     DIOPI_BOUND(diopiFusedAddRootMeanSquareNormInp),
     DIOPI_BOUND(diopiFusedDecoderAttentionInp),
+    {"scratch_peak", scratchPeakOf, METH_NOARGS, "Most bytes of scratch that calls on torch's current stream have held at a time."},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "diopi_torch", "The DIOPI operators on torch tensors.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -275,6 +275,9 @@ class Context:
     def clear_tensors(self) -> None:
         self._rt.diopirtContextClearTensors(self.handle)
 
+    def before_event(self) -> None:
+        """Orders the stream behind what an event recorded on this context stands for."""
+
     @property
     def scratch_peak(self) -> int:
         return int(self._rt.diopirtContextScratchPeak(self.handle))
@@ -337,6 +340,7 @@ class Event:
             raise DiopiException("hipEventCreate failed")
 
     def record(self, ctx: Context) -> None:
+        ctx.before_event()
         if self._rt.diopirtEventRecord(self.handle, ctx.handle) != 0:
             raise DiopiException("hipEventRecord failed")
 
@@ -356,12 +360,22 @@ class Event:
 
 
 class _DefaultContext(Context):
-    """The functions that get no context run on torch's current stream: waiting for this context waits for them too."""
+    """Stands for the functions that get no context, wherever they run: on torch's current stream, whichever that was.  Waiting for
+    this context waits for all of them; an event recorded on it comes after those on the stream that is current then.  Their
+    scratch is torch's, and scratch_peak has it too; malloc_count is this context's own pool's alone."""
 
     def synchronize(self) -> None:
         super().synchronize()
         if torch.cuda.is_available():
-            torch.cuda.current_stream().synchronize()
+            torch.cuda.synchronize()  # they may have run on any stream, from any thread
+
+    def before_event(self) -> None:
+        if self.torch_stream is not None:
+            self.torch_stream.wait_stream(torch.cuda.current_stream())
+
+    @property
+    def scratch_peak(self) -> int:
+        return max(super().scratch_peak, torch_ops().scratch_peak())
 
 
 _default_ctx = None

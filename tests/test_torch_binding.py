@@ -112,3 +112,37 @@ def test_context_on_torchs_default_stream():
         seen = cache.clone()
         assert float(seen[1, 0, 0]) == n and float(seen[1, 0, 63]) == n
     ctx.close()
+
+
+def _long_call():
+    """Attention that takes milliseconds, without a context."""
+    q = torch.randn(1, 8192, 16, 128, device=DEV).half()
+    F.flash_attention(q, q, q, None, 0.0, None, False)
+    torch.cuda.synchronize()
+    return lambda: F.flash_attention(q, q, q, None, 0.0, None, False)
+
+
+@pytest.mark.gpu
+def test_the_default_context_stands_for_calls_without_a_context():
+    ctx, call = rt.default_context(), _long_call()
+    torch_events, events = [torch.cuda.Event(enable_timing=True) for _ in range(2)], [rt.Event() for _ in range(2)]
+    torch_events[0].record()
+    events[0].record(ctx)
+    for _ in range(5):
+        call()
+    events[1].record(ctx)
+    torch_events[1].record()
+    torch.cuda.synchronize()
+    whole = torch_events[0].elapsed_time(torch_events[1])
+    assert 0.5 * whole <= events[0].elapsed_ms(events[1]) <= 1.01 * whole + 0.1, whole  # host gaps are on both sides
+    # calls on another stream, waited for outside of it
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            call()
+    assert not stream.query()  # tens of milliseconds of work
+    ctx.synchronize()
+    assert stream.query()
+    # their scratch: partial sums of two ranges for three sequences and eight heads of 128
+    _step(*_inputs(25))
+    assert ctx.scratch_peak >= 3 * 2 * 8 * 130 * 4
