@@ -1,5 +1,8 @@
 """The builtin functions that hand torch tensors to the operators (diopi_amd/csrc/rt/torch_binding.cpp): what they refuse, and
 that calls without a context keep the order of torch's current stream, whatever the thread, stream or graph."""
+import os
+import subprocess
+import sys
 import threading
 
 import pytest
@@ -29,6 +32,17 @@ def test_arguments_that_are_no_tensors_of_a_known_type():
         F.rms_norm_backward([None], x, w, None, (4,), 1e-6, inv_rms=torch.ones(2))
     with pytest.raises(rt.DiopiException, match="rank 9"):
         F.destindex_copy_kv(torch.ones([1] * 9), torch.zeros(1, dtype=torch.int32), torch.ones([1] * 9))
+
+
+def test_a_build_of_the_c_libraries_alone(tmp_path):
+    for path in (rt.RT_LIB_PATH, rt.IMPL_LIB_PATH):
+        os.symlink(path, tmp_path / os.path.basename(path))
+    code = ("import torch; from diopi_amd import functions as F, runtime as rt\n"
+            "try: F.rms_norm(torch.ones(2, 4), (4,), torch.ones(4), None, 1e-6)\n"
+            "except rt.DiopiException as e: print(e)")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", code], cwd=root, env=dict(os.environ, DIOPI_AMD_LIB_DIR=str(tmp_path)), capture_output=True, text=True, timeout=100)
+    assert "device memory" in res.stdout, res.stderr[-2000:]
 
 
 def _step(w, x, go, weight):
@@ -146,3 +160,20 @@ def test_the_default_context_stands_for_calls_without_a_context():
     # their scratch: partial sums of two ranges for three sequences and eight heads of 128
     _step(*_inputs(25))
     assert ctx.scratch_peak >= 3 * 2 * 8 * 130 * 4
+
+
+@pytest.mark.gpu
+def test_the_ctypes_route_gives_the_same(monkeypatch):
+    args = _inputs(26)
+    want = _step(*args)
+    x = torch.randn(300, 4, 64, device=DEV).half()
+    cu = torch.tensor([0, 100, 300], dtype=torch.int32, device=DEV)
+    attend = lambda: (F.flash_attention_varlen(x, x, x, cu, cu, None, 200, 200, 0.0, None, True), F.GLOBAL_STATE["flash_attention_varlen_softmax_lse"])
+    hidden, weight = torch.randn(2, 256, device=DEV).half(), torch.randn(256, 768, device=DEV).half() * 0.05
+    caches, lens = [torch.zeros(1, 2, 2, 33, 128, device=DEV).half() for _ in range(2)], torch.tensor([3, 9], dtype=torch.int32, device=DEV)
+    fused = lambda: F.fused_decoder_attention_inp(hidden.clone(), weight, None, None, 0, *caches, None, 32 - lens, lens, 33, 0, 2, 2, 128, 33, 128, 10000.0)
+    want += attend() + (fused(),)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(rt, "_torch_ops", rt._CtypesOps())
+    for n, (a, b) in enumerate(zip(_step(*args) + attend() + (fused(),), want)):
+        assert_bit_equal(a, b, f"output {n}")
