@@ -45,6 +45,14 @@ def test_a_build_of_the_c_libraries_alone(tmp_path):
     assert "device memory" in res.stdout, res.stderr[-2000:]
 
 
+def test_the_c_libraries_are_made_without_python(tmp_path):
+    """`make all` asks for nothing that needs torch's headers or Python's."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(rt.__file__)), "csrc")
+    res = subprocess.run(["make", "-C", csrc, "-n", "-B", "all"], capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0 and "libdiopi_impl.so" in res.stdout
+    assert "torch" not in res.stdout and "python" not in res.stdout.lower()
+
+
 def _step(w, x, go, weight):
     """Three operators that take scratch, without a context."""
     inv = torch.rsqrt((x * x).mean(-1) + 1e-6)
