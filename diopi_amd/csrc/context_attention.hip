@@ -29,11 +29,11 @@
 //
 // Heads of 64 have a kernel of their own, ctxAttn64, on the same tiles and layouts.
 //
-// The same kernels serve diopiFlashAttentionVarLen (proto/include/diopi/functions_ext.h:355-359; Python statement
+// The same operator code serves diopiFlashAttentionVarLen (proto/include/diopi/functions_ext.h:355-359; Python statement
 // customized_test.py:525-588 with multi_head_attention_inside, 36-57): sequences given by cumulative lengths, G query
 // heads per key/value head, an explicit softmax scale, causal or full attention, and the row-wise log-sum-exp as a
-// second output.  That form is a template flag (GEN): the lightllm operator keeps its literal scale and its
-// compile-time causal structure.
+// second output.  With heads of 128 that form (GEN at the launchers) is ctxAttnMfma's; the lightllm operator has ctxAttnPipe,
+// with a literal scale and a compile-time causal structure.
 #include <cmath>
 #include <cstdlib>
 #include <mutex>
@@ -252,13 +252,11 @@ __device__ __forceinline__ int4 ctxAttnItem(const CtxArgs& a, int p, int bm) {
     return a.plan != nullptr ? a.plan[p] : ctxAttnTileAt(a, p, bm);
 }
 
-template <typename T, int NWV, bool GEN>
+template <typename T, int NWV>
 __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnMfma(T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                                CtxArgs a) {
-    // exp(x / sqrt(D)) = exp2(x * log2(e) / sqrt(D)): one literal factor (a run-time one in the general form)
-    constexpr float kScaleLog2 = 0.12751743082459868f;  // log2(e) / sqrt(128)
-    const float scaleLog2 = GEN ? a.scaleLog2 : kScaleLog2;
-    const bool causal = GEN ? a.causal : true;
+    const float scaleLog2 = a.scaleLog2;
+    const bool causal = a.causal;
     using Ops = Mfma32<T>;
     using Frag = typename Ops::Frag;
     constexpr int BM = NWV * 32;  // query rows per work-group: each of the NWV waves owns 32 of them
@@ -287,8 +285,8 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnMfma(T* 
     const int n = lane % 32;   // query column of this lane in every accumulator
     const int hh = lane / 32;  // which half of the k slots / which 4-row sub-block of the accumulator
     const int64_t qPitch = static_cast<int64_t>(a.H) * kHD;                   // row pitch of q and out
-    const int64_t rowPitch = GEN ? static_cast<int64_t>(a.H / a.G) * kHD : qPitch;  // row pitch of k and v
-    const int kvHead = GEN ? head / a.G : head;
+    const int64_t rowPitch = static_cast<int64_t>(a.H / a.G) * kHD;  // row pitch of k and v
+    const int kvHead = head / a.G;
     const T* qBase = q + si.start * qPitch + static_cast<int64_t>(head) * kHD;
     const T* kBase = k + si.start * rowPitch + static_cast<int64_t>(kvHead) * kHD;
     const T* vBase = v + si.start * rowPitch + static_cast<int64_t>(kvHead) * kHD;
@@ -296,10 +294,10 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnMfma(T* 
     // ---- Q fragments (B operand of S^T): row = m0 + 32*wave + n, k slot (hh, e) <-> dim 16*s + 8*hh + e ----
     // The query is multiplied by softmax_scale * log2(e) here, once, so that the first product delivers the exponent
     // of 2 directly.  That rounds the scaled query to the element type, the size of the rounding the reference applies
-    // to its scores (functions_lightllm.cpp:121 keeps them in the tensor dtype).  The general form with bf16 tensors
-    // (8 bits) does not: it also returns the log-sum-exp, which would inherit that rounding; it keeps the
-    // multiplication in fp32, one instruction per score, and sums the unrounded probabilities.
-    constexpr bool kFold = std::is_same<T, half_t>::value || !GEN;
+    // to its scores (functions_lightllm.cpp:121 keeps them in the tensor dtype).  With bf16 tensors (8 bits) it is not: the
+    // log-sum-exp, which is returned too, would inherit that rounding; the multiplication stays in fp32, one instruction
+    // per score, and the row sum takes the unrounded probabilities.
+    constexpr bool kFold = std::is_same<T, half_t>::value;
     const float toLog2 = kFold ? 1.f : scaleLog2;  // from the unit of the score accumulators to powers of two
     const int qRow = m0 + wave * 32 + n;
     const int qRowLd = qRow < L ? qRow : L - 1;
@@ -550,15 +548,12 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnMfma(T* 
     // ---- normalise, transpose through LDS, write rows with 16-byte stores ----
     const float lTot = lRun + __shfl_xor(lRun, 32, kWave);
     const float inv = 1.0f / lTot;
-    if constexpr (GEN) {
-        // ln sum_j exp(scale * s_j) = ln 2 * (reference maximum in log2 units + log2 of the sum relative to it)
-        if (a.lse != nullptr && hh == 0 && qRow < L && qRow < a.lseStride)
-            a.lse[(static_cast<int64_t>(planned.x) * a.H + head) * a.lseStride + qRow] = 0.6931471805599453f * (mRun * toLog2 + __builtin_amdgcn_logf(lTot));
-    }
+    // ln sum_j exp(scale * s_j) = ln 2 * (reference maximum in log2 units + log2 of the sum relative to it)
+    if (a.lse != nullptr && hh == 0 && qRow < L && qRow < a.lseStride)
+        a.lse[(static_cast<int64_t>(planned.x) * a.H + head) * a.lseStride + qRow] = 0.6931471805599453f * (mRun * toLog2 + __builtin_amdgcn_logf(lTot));
     waitLdsLoads();
     __syncthreads();  // the K/V tiles are dead and no request is in flight; reuse the storage as a [BM][kLD] output tile
     T* sO = smem;
-    static_assert(kHD == 128, "scaleLog2 is written out for head size 128");
 #pragma unroll
     for (int mb = 0; mb < kHD / 32; ++mb) {
 #pragma unroll
@@ -1139,9 +1134,11 @@ struct Special {
     }
 };
 
-template <typename T, int NWV>
-__global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 3 : 2) void ctxAttn64(T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k,
-                                                                          const T* __restrict__ v, CtxArgs a) {
+constexpr int kWaves64 = 4;  // waves of a work-group
+template <typename T>
+__global__ __launch_bounds__(kWaves64* kWave, 3) void ctxAttn64(T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
+                                                                CtxArgs a) {
+    constexpr int NWV = kWaves64;
     using Ops = Mfma32<T>;
     using Frag = typename Ops::Frag;
     constexpr int D = 64;
@@ -1575,10 +1572,11 @@ diopiError_t launchMfma(diopiContextHandle_t ctx, hipStream_t stream, void* out,
     constexpr int ldsBytes = (kStaging > kOutTile ? kStaging : kOutTile) * static_cast<int>(sizeof(T));
     auto kernel = [] {
         if constexpr (HD == 64) {
-            return ctxAttn64<T, NWV>;
+            static_assert(NWV == kWaves64, "the one shape that ctxAttn64 has");
+            return ctxAttn64<T>;
         } else if constexpr (GEN) {
-            return ctxAttnMfma<T, NWV, true>;
-        } else {  // the lightllm operator: causal, one key/value head per query head, the literal scale
+            return ctxAttnMfma<T, NWV>;
+        } else {  // causal, one key/value head per query head, the literal scale
             return ctxAttnPipe<T, NWV>;
         }
     }();
