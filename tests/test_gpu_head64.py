@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from diopi_amd import functions as F
+from diopi_amd import runtime as rt
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -245,11 +246,40 @@ def test_attention_scale_that_fp32_holds_as_zero():
 
 def test_attention_where_no_plan_can_be_had():
     """The allocation-free entry point with more query tiles than its static plan holds: refused for heads of 128, for heads of 64
-    the general kernel takes the call, as it did every one."""
-    lens = [3, 70, 2] * 2800
-    q, k, v, start = _packed(lens, 1, 1, torch.float16, 7)
-    loc, length = (torch.tensor(t, dtype=torch.int32, device=DEV) for t in (start[:-1].tolist(), lens))
-    out = F.context_attention_no_alloc(q, k, v, torch.zeros_like(q), loc, length, 70)
-    torch.cuda.synchronize()
-    want = F.context_attention(q, k, v, torch.zeros_like(q), loc, length, 70)
-    assert ((out - want).abs() <= 3 * 2.0 ** -11 * want.abs() + 1e-4).all()
+    the general kernel takes the call, as it did every one.  From a context the same call takes its plan and the tile kernel."""
+    lens = [10490 + i % 3 for i in range(100)]  # 8203 tiles of 128 rows and 100 sequences, against 8192
+    total = sum(lens)
+    assert (total + 127) // 128 + len(lens) > 8192
+    assert (4 * len(lens) + total // 128 + 1) * 4 <= 65536  # what a plan takes in LDS: the tile kernel is not ruled out before
+    start = np.concatenate(([0], np.cumsum(lens)))[:-1]
+    loc, length = (torch.tensor(t, dtype=torch.int32, device=DEV) for t in (start.tolist(), lens))
+    g = torch.Generator(device=DEV).manual_seed(7)
+    q, k, v = (torch.randn(total, 1, 64, generator=g, device=DEV).half() for _ in range(3))
+    out = F.context_attention_no_alloc(q, k, v, torch.zeros_like(q), loc, length, max(lens))
+    want = F.context_attention(q, k, v, torch.zeros_like(q), loc, length, max(lens))
+    # both round a result once; before that the scores' fp32 sums, taken in other orders, move it by 2^-14 of values of up to 5
+    assert ((out - want).abs() <= 2 * 2.0 ** -11 * want.abs() + 10 * 2.0 ** -14).all()
+    assert not torch.equal(out, want)  # two kernels
+    wide = torch.zeros(2500 * 304, 1, 128, dtype=torch.float16, device=DEV)
+    many = torch.arange(2500, dtype=torch.int32, device=DEV) * 304
+    with pytest.raises(rt.DiopiException, match="at most 8192"):
+        F.context_attention_no_alloc(wide, wide, wide, torch.zeros_like(wide), many, torch.full_like(many, 304), 304)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("batch,longest", [(33, 300), (64, 300), (64, 20), (100, 300), (40, 1100), (1, 33000)])
+def test_attention_over_many_tiles(batch, longest, causal, D):
+    """Tiles that the work-groups find (up to 64 sequences, of which the later ones stand in the upper half of a ballot, and 256 tiles)
+    and tiles from a table, of lengths in no order, some of them zero or the same."""
+    H = 1 if batch == 1 else 3
+    lens = [longest] if batch == 1 else [(i * 37) % longest + 1 if i % 7 else (0 if i % 2 else longest) for i in range(batch)]
+    g = torch.Generator().manual_seed(batch + D)
+    q, k, v = (torch.randn(sum(lens), H, D, generator=g).half().to(DEV) for _ in range(3))
+    cu = torch.tensor(np.concatenate(([0], np.cumsum(lens))), dtype=torch.int32, device=DEV)
+    call = lambda vv: (F.flash_attention_varlen(q, k, vv, cu, cu, None, longest, longest, 0.0, None, causal), F.GLOBAL_STATE["flash_attention_varlen_softmax_lse"])
+    (out, lse), (general, general_lse) = call(v), call(_unaligned(v))
+    # heads of 128 round the scaled query and the probabilities to 16 bits: scores of up to 6, values of up to 5
+    slack = 2.0 ** -11 * (6 + 1) * 5 if D == 128 else 10 * 2.0 ** -14
+    assert ((out - general).abs() <= 2 * 2.0 ** -11 * general.abs() + slack).all()
+    assert ((lse - general_lse).abs() <= (6 * 2.0 ** -10 if D == 128 else 1e-5) + 1e-6 * general_lse.abs()).all()

@@ -683,9 +683,9 @@ def test_decode_gqa_config5_scaled():
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 def test_decode_head_size_64(dtype):
-    """Head size 64 takes the matrix-core kernel that reads its operands straight from the cache rows (score operator)
-    and the shape-agnostic reduce kernel: one query head per cache head and grouped heads, ragged lengths that are no
-    multiple of 16 or 128 (and an empty sequence), 32- and 64-bit index tensors."""
+    """Head size 64 takes the matrix-core kernels of head size 128, two neighbouring heads to a 256-byte piece of a cache row:
+    one query head per cache head and grouped heads, an odd number of cache heads, ragged lengths that are no multiple of 16 or
+    128 (and an empty sequence), 32- and 64-bit index tensors."""
     dt = TORCH_DTYPES[dtype]
     for (H, Hkv, idt) in ((8, 8, torch.int32), (12, 3, torch.int64), (16, 1, torch.int32)):
         lens = np.array([1, 15, 16, 17, 0, 127, 128, 129, 300, 77], dtype=np.int64)
