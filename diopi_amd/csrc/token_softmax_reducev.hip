@@ -582,9 +582,11 @@ diopiError_t launchWave(diopiContextHandle_t ctx, hipStream_t stream, void* out,
     sp.ranked = pieces * a.batch * sp.splits >= 2 * numCU;
     // Waves of a work-group: 16 where there are fewer work-groups than compute units, for what a unit has in flight then is what one
     // work-group has (4 and 16 waves: one sequence of 4000 tokens with 8 kv heads of 4 query heads 24.4 and 18.5 us, 8 of 500..2000
-    // with the same heads 21.9 and 16.1, one of 700 with 32 heads 7.0 and 6.4, 2 of 20001 and 50001 with 8 of 8 (144 work-groups) 55.1
-    // and 42.0; one of 16000 with 40 heads (320) 39.0 and 40.7, 16 of 100..1000 with 32 (512) 17.2 and 19.4)
-    const bool wide = groups() < numCU;
+    // with the same heads 21.9 and 16.1, one of 700 with 32 heads 9.0 and 7.1, 2 of 20001 and 50001 with 8 of 8 (144 work-groups) 55.1
+    // and 42.0; one of 16000 with 40 heads (320) 39.0 and 40.7, 16 of 100..1000 with 32 (512) 17.2 and 19.4).  A window of no more
+    // sub-tiles than four waves take in one turn has nothing for the others but a part in the hand-over (8 kv heads of 8 query heads, one
+    // sequence of 64 tokens 6.4 and 8.4 us, of 400 7.5 and 9.6; of 520, five sub-tiles, 10.8 and 10.3)
+    const bool wide = groups() < numCU && a.maxInputLen > kRvWaves * kSub;
     const dim3 grid(static_cast<unsigned>(pieces), static_cast<unsigned>(a.batch), static_cast<unsigned>(sp.splits));
     auto launch = [&](auto groupTag, auto wavesTag) -> diopiError_t {
         constexpr int GC = decltype(groupTag)::value, NW = decltype(wavesTag)::value;

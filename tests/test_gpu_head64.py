@@ -19,7 +19,7 @@ def _unaligned(t):
     return out.copy_(t)
 
 
-def _decode(lens, H, Hkv, dt, idt, seed):
+def _decode(lens, H, Hkv, dt, idt, seed, D=64):
     g = torch.Generator().manual_seed(seed)
     B, longest, total = len(lens), max(lens) + 5, sum(lens)
     slots = total + 3
@@ -29,7 +29,7 @@ def _decode(lens, H, Hkv, dt, idt, seed):
         b_loc[i, longest - n:] = order[start[i]:start[i] + n].to(idt)
     rand = lambda *shape: torch.randn(*shape, generator=g).to(dt).to(DEV)
     return dict(B=B, longest=longest, total=total, start=start, b_loc=b_loc.to(DEV), b_start=torch.from_numpy(start).to(idt).to(DEV),
-                b_len=torch.tensor(lens, dtype=idt, device=DEV), q=rand(B, H, 64), k=rand(slots, Hkv, 64), v=rand(slots, Hkv, 64), logits=rand(H, total) * 3)
+                b_len=torch.tensor(lens, dtype=idt, device=DEV), q=rand(B, H, D), k=rand(slots, Hkv, D), v=rand(slots, Hkv, D), logits=rand(H, total) * 3)
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
@@ -59,6 +59,24 @@ def test_softmax_reducev(dt, H, Hkv, idt):
         bound = (u + n * 2.0 ** -23) * sizes + n * tiny * v.abs().amax(1) + u * want.abs() + tiny + 1e-6
         assert ((out[i].double() - want).abs() <= 1.01 * bound).all(), (i, n)
         assert ((out[i].double() - general[i].double()).abs() <= 2.02 * bound).all(), (i, n)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Hkv,lens", [(16, 2, [1, 128, 129, 507]), (16, 2, [1, 384, 385, 508]), (9, 3, [508]), (32, 32, [700, 3, 699, 0, 513, 129, 1, 600, 64])])
+def test_softmax_reducev_waves_and_order(H, Hkv, lens, D):
+    """Few work-groups over windows of 512 and of 513 columns, which four and sixteen waves take, and more work-groups than compute
+    units over sequences of unequal length, which are taken longest first."""
+    w = _decode(lens, H, Hkv, torch.float16, torch.int32, 264 + H, D)
+    out = torch.full((w["B"], H, D), 5.0, dtype=torch.float16, device=DEV)
+    F.token_softmax_reducev(w["logits"], w["v"], out, w["b_loc"], w["b_start"], w["b_len"], w["longest"], 0)
+    u, tiny = ROUND[torch.float16]
+    for i, n in enumerate(lens):
+        at = int(w["start"][i])
+        v = w["v"][w["b_loc"][i, w["longest"] - n:].long()].double().repeat_interleave(H // Hkv, 1).transpose(0, 1).contiguous() if n else torch.zeros(H, 1, D, device=DEV).double()
+        p = torch.softmax(w["logits"][:, at:at + n].double(), -1) if n else torch.zeros(H, 1, device=DEV).double()
+        want, sizes = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
+        bound = (u + n * 2.0 ** -23) * sizes + n * tiny * v.abs().amax(1) + u * want.abs() + tiny + 1e-6  # as above
+        assert ((out[i].double() - want).abs() <= 1.01 * bound).all(), (i, n)
 
 
 def test_softmax_reducev_infinite_values():
