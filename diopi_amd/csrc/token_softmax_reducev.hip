@@ -576,10 +576,13 @@ diopiError_t launchWave(diopiContextHandle_t ctx, hipStream_t stream, void* out,
     }
     ROCM_CHECK(a.batch <= 65535, "batch %d exceeds the launch limit of 65535 sequences", a.batch);
     ROCM_CHECK(sp.splits <= 65535, "max_input_len %d needs more than 65535 ranges of %d tokens", a.maxInputLen, TT);
-    // Work-groups that all start at once need no order, and finding an item's rank is one of the longer steps of a short one: one
-    // sequence of 4000 tokens (16 work-groups) 20.0 us ranked and 18.5 not, 16 of 100..1000 (512) 18.0 and 17.2, 64 of 512..2048
-    // with 8 kv heads of 8 query heads (512) 40.1 and 41.4
-    sp.ranked = pieces * a.batch * sp.splits >= 2 * numCU;
+    // Work-groups that have a compute unit each need no order, and finding an item's rank is one of the longer steps of a short one:
+    // one sequence of 4000 tokens (16 work-groups) 20.0 us ranked and 18.5 not, 24 of 128..3001 with 8 kv heads of 4 query heads (192)
+    // 24.8 and 23.1.  Where some units get two, an order keeps the long ones apart (8 of 500..2000 with 40 heads (320): 26.7 and 29.0,
+    // 10 of 100..2000 with the same (400) 27.0 and 29.6, with 32 heads (320) 24.6 and 26.1), unless all are short (8 of 60..128 with 40
+    // heads 7.6 and 6.1) or as long as each other (12 of 2000 with 32 heads 38.3 and 36.8), which the host cannot see.
+    // With heads of 64 a launch of that size is not ranked: its ranges are short
+    sp.ranked = pieces * a.batch * sp.splits >= 2 * numCU || (HD == kD && groups() > numCU && a.maxInputLen > kRvWaves * kSub);
     // Waves of a work-group: 16 where there are fewer work-groups than compute units, for what a unit has in flight then is what one
     // work-group has (4 and 16 waves: one sequence of 4000 tokens with 8 kv heads of 4 query heads 24.4 and 18.5 us, 8 of 500..2000
     // with the same heads 21.9 and 16.1, one of 700 with 32 heads 9.0 and 7.1, 2 of 20001 and 50001 with 8 of 8 (144 work-groups) 55.1
