@@ -70,7 +70,7 @@ __device__ __forceinline__ Frag zeroFrag() {
 //   * 16 consecutive lanes read one piece (256 contiguous bytes) of one token; a wave owns HW
 //     adjacent pieces, so it reads HW*256 contiguous bytes per token and the waves of a work-group
 //     cover adjacent pieces of the same tokens;
-//   * the loads a lane issues per unit (TU = UNIT/HW tokens x HW pieces: 16 loads for UNIT = 64, 4 for UNIT = 16; the launcher
+//   * the loads a lane issues per unit (TU = UNIT/HW tokens x HW pieces: 16 loads for UNIT = 64, 8 for 32, 4 for 16; the launcher
 //     says which) are all in flight before the first use; each [16 tokens x 128 dims] block then goes through a wave-private LDS tile
 //     (row pitch 272 bytes: conflict-free for both the 16-byte row writes and the 16-byte
 //     column-block reads) and comes back in the MFMA B-operand layout;
@@ -333,8 +333,14 @@ diopiError_t launchStaged(hipStream_t stream, void* out, const void* q, const vo
     // Loads a lane has in flight per unit of tokens: 16 with one query head per kv head; with grouped heads 4, where the rows
     // compete with the logits being written (128 sequences of 1024..8192 tokens, 8 kv heads of 8 query heads: 234.3 us against
     // 242.9 with 16 and 243.6 with 8; with one query head per kv head 4 and 8 are 1 % slower than 16), unless work-groups are too
-    // few to compete with anything and what counts is how long one takes (the first two shapes above: 6.6 -> 4.8 and 7.6 -> 6.7 us)
-    if (a.G == 1 || fewGroups) {
+    // few to compete with anything and what counts is how long one takes: then as many as give each of the waves that take the tokens
+    // of a piece in turn a unit of a tile of 64 (one wave, four or more pieces: the first two shapes above 6.6 -> 4.8 and 7.6 -> 6.7 us;
+    // two waves, 2 kv heads of 8 query heads: one sequence of 64 tokens 3.79 us with 16 loads a lane and 3.28 with 8, of 4000 4.09 and
+    // 3.69, and 0.5 more than with 16 with 4; four waves, one kv head of 8: 64 tokens 4.3 with 16 and 3.6 with 4)
+    if (a.G > 1 && fewGroups && HS == 2) {
+        hipLaunchKernelGGL((tokenAttStaged<T, HD, HW, 32>), grid, dim3(kAttThreads), outLds, stream, static_cast<T*>(out), static_cast<const T*>(q),
+                           static_cast<const T*>(k), a, TT, HS, scale, order);
+    } else if (a.G == 1 || (fewGroups && HS == kAttWaves)) {
         hipLaunchKernelGGL((tokenAttStaged<T, HD, HW, 64>), grid, dim3(kAttThreads), outLds, stream, static_cast<T*>(out), static_cast<const T*>(q),
                            static_cast<const T*>(k), a, TT, HS, scale, order);
     } else {
