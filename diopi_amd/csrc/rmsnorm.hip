@@ -693,12 +693,11 @@ diopiError_t launchBwdFused(diopiContextHandle_t ctx, hipStream_t stream, const 
     if (d.n2 % EPV != 0 || d.n2 > INT32_MAX) return diopiSuccess;
     const int64_t nvec = d.n2 / EPV;
     // The shape of the work-groups by the packets a thread holds per row (NVT), all within 128 KiB of LDS per compute unit
-    // (a team array is NVT * 256 packets of ColAcc).  Measured without grad_bias, main kernel alone:
+    // (a team array is NVT * 256 packets of ColAcc).  Measured without grad_bias, main kernel alone, two groups of two teams against
+    // one group of four:
     //   fp32 [32768, 1024] (NVT 1): 67.5 against 63.4 us; bf16 [8192, 4096] (NVT 2): 37.8 against 36.7 us
-    //   bf16 [4096, 8192] (NVT 4): one group of two teams 46.3 us against 108.9 us for four teams, whose 16 waves leave a lane
-    //   128 registers where the kernel wants 217
-    // so fewer packets than four take one group of four teams; fp32 rows of up to 8192 columns
-    // (NVT 8, 64 KiB per team array, 236 registers) one group of two.  With grad_bias a team has two arrays: one group of two
+    // so one or two packets take one group of four teams; fp32 rows of up to 8192 columns (NVT 8, 64 KiB per team array, 236 registers)
+    // take one group of two.  With grad_bias a team has two arrays: one group of two
     // teams (one of one team at NVT 8).  Wider teams where they pay: see below.
     constexpr int kMaxNvt = sizeof(T) == 4 ? 8 : 4;
     if (nvec > static_cast<int64_t>(kMaxNvt) * kBwdTeam) return diopiSuccess;
@@ -719,20 +718,22 @@ diopiError_t launchBwdFused(diopiContextHandle_t ctx, hipStream_t stream, const 
     const bool wideBias = gBias != nullptr && nvc == 4 && sizeof(T) == 4;
     // Teams of the width of a row, in waves, where idle threads or too few rows under way cost most (us for the whole operator,
     // teams of 256 -> teams of that width):
-    //   rows of up to 128 packets, 16 teams of 64 or 8 of 128: bf16 [30000, 512] 34.4 -> 21.6, [12000, 800] 19.2 -> 16.4, fp32
-    //   [30000, 256] 29.0 -> 21.2, [12000, 512] 18.6 -> 18.6 (129 to 192 packets in 5 teams of 192 lose: bf16 [3900, 1440] 13.7 -> 14.3)
+    //   rows of up to 128 packets, more than a row for each of four teams a compute unit, 16 teams of 64 or 8 of 128: bf16 [30000, 512]
+    //   34.4 -> 21.6, [12000, 800] 19.2 -> 16.4, [1237, 512] 8.3 -> 7.2, fp32 [30000, 256] 29.0 -> 21.2, [12000, 512] 18.6 -> 18.6 (fewer
+    //   rows gain nothing or lose: bf16 [64, 512] 6.7 -> 6.9, fp32 [300, 512] 6.5 -> 6.6; 129 to 192 packets in 5 teams of 192 lose: bf16 [3900, 1440] 13.7 -> 14.3)
     //   257 to 512 packets and few rows, one packet a thread: bf16 [1237, 2560] 13.0 -> 11.6, [1237, 4096] 15.6 -> 14.8 (3900 rows of
     //   2560 lose: 17.3 -> 18.9)
     //   513 to 1024 packets and few rows, two teams of two packets a thread: bf16 [1237, 5120] 18.1 -> 16.5, [3900, 5120] 29.6 -> 28.3,
     //   fp32 [300, 4096] 12.5 -> 10.6, [2500, 4096] 28.1 -> 27.0
-    const bool fits = gBias == nullptr && !wide && (nvec <= 128 || (nvec > 256 && nvec <= 512 && d.n1 < 8 * static_cast<int64_t>(deviceInfo().numCU)) ||
+    const int64_t numCU = deviceInfo().numCU;
+    const bool fits = gBias == nullptr && !wide && ((nvec <= 128 && d.n1 > 4 * numCU) || (nvec > 256 && nvec <= 512 && d.n1 < 8 * numCU) ||
                                                     (nvec > 512 && nvec <= 1024));
     const int fitting = !fits ? 0 : static_cast<int>(ceilDiv(nvec, (nvec > 512 ? 2 : 1) * kWave)) * kWave;  // threads of such a team
     // teams of a work-group: each owns rows of its own
     const int groups = fits ? (nvec <= 128 ? 1024 / fitting : (nvec <= 320 ? 3 : 2))
                             : (wide ? (nvec <= 512 ? 2 : 1) : (wideBias ? 1 : (gBias ? (nvc == 8 ? 1 : 2) : (nvc <= 2 ? 4 : 2))));
     // as many work-groups as there are compute units (fewer when there are not enough rows to give every team one)
-    const int64_t maxBlocks = deviceInfo().numCU;
+    const int64_t maxBlocks = numCU;
     const int teamsPerGroup = groups;
     const int numParts = static_cast<int>(std::min<int64_t>(maxBlocks, ceilDiv(d.n1, teamsPerGroup)));
     const int n2 = static_cast<int>(d.n2);
