@@ -84,7 +84,6 @@ struct PlanStore {
 
 // Tile plans of the allocation-free entry point.  One array per device the library runs on, held until the process
 // ends; every call on a device shares it, so such calls must not overlap on one device.
-constexpr int kScannedTiles = 256;  // most query tiles of a call whose work-groups look for theirs one tile count after the other
 constexpr int kStaticPlanEntries = 8192;  // 128 KiB: query tiles + sequences of one call
 static __device__ __align__(256) int4 scratch[kStaticPlanEntries];
 
@@ -220,6 +219,8 @@ __global__ __launch_bounds__(kPlanThreads) void ctxAttnPlan(int4* __restrict__ p
         }
     }
 }
+
+constexpr int kScannedTiles = 256;  // most query tiles of a call whose work-groups look for theirs one tile count after the other
 
 // The same visiting order without a table, for up to kWave sequences (one per lane): the entry at position p, found by every wave for
 // itself.  Causal: tile indices from the highest down, the sequences that have such a tile at each.  Full attention, where a
@@ -1536,12 +1537,14 @@ diopiError_t launchMfma(diopiContextHandle_t ctx, hipStream_t stream, void* out,
     }
     ROCM_CHECK(total < INT32_MAX / 2, "context attention: too many tiles for one launch");
     a.totalItems = static_cast<int>(total);
-    // Work-groups that find their tiles themselves take about 0.8 us longer each, so a table pays for itself once they follow
-    // each other often enough on a compute unit, the sooner the fewer fit there side by side: 8-wave groups one (8 prompts of
-    // 1024..4096 rows, 11 in a row: 557 us with the table, 569 without), 4-wave groups two (24 of 16..300 rows, up to 3.4 in a row:
-    // 43.4 and 36.8) or, with heads of 64, three (8 of 100..2560 rows, up to 4.5 in a row: 267 and 255).
-    constexpr int kSideBySide = NWV == 8 ? 1 : (HD == 64 ? 3 : 2);
-    const bool table = a.batch > kWave || a.tilesBound > kScannedTiles || total > (NWV == 8 ? 3 : 5) * kSideBySide * static_cast<int64_t>(deviceInfo().numCU);
+    // Work-groups that find their tiles themselves take about 0.8 us longer each, which a table pays back only where nothing else runs
+    // on a compute unit meanwhile (8-wave groups, one to a unit) and many follow each other there (us, 32 heads of 128, causal, with and
+    // without the table: 2 prompts of 1024..3000 rows, 2.2 in a row, 114 and 111, 4 of them, 4.5, 181.2 and 180.0, 5, 5.6, 207.5 and
+    // 208.7, 6, 6.8, 249 and 256, 8 of 1024..4096, 11, 524 and 534).  Full attention is better off without one at any length, as the
+    // order that is found there goes by length (8 of 100..2560, 32 and 64 heads on 8: 344 and 329, 669 and 643), and so are 4-wave groups,
+    // of which two or, with heads of 64, three share a unit (24 of 16..300 rows 37.7 and 31.6, 64 of them 95.5 and 82.2, with heads of
+    // 64 63.4 and 49.0; 10 of 100..2560, 64 heads of 64 on 8, 611 and 593, causal 337 and 337).
+    const bool table = a.batch > kWave || a.tilesBound > kScannedTiles || (NWV == 8 && a.causal && total > 5 * static_cast<int64_t>(deviceInfo().numCU));
     // visiting order of the query tiles, rebuilt by every call on the device: context-owned scratch, or the library's
     // static array when the caller must not allocate.  With heads of 128 the memory is asked for with and without a table, so that
     // what a call needs of its context does not hang on its size.
