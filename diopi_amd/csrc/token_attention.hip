@@ -310,9 +310,10 @@ diopiError_t launchStaged(hipStream_t stream, void* out, const void* q, const vo
     while (shortest < longest && ceilDiv(a.maxInputLen, shortest) > 65535) shortest *= 2;
     if (TT < shortest) TT = shortest;
     const int gridX = static_cast<int>(ceilDiv(pieces, HS * HW));
-    // Shorter tiles where those leave compute units idle, until there are two work-groups for each (256 and 64 tokens: one
-    // sequence of 4000 tokens with 8 kv heads of 4 query heads 16.4 and 6.6 us, 8 of 500..2000 with the same heads 18.3 and 7.6,
-    // 24 of 128..3001 with heads of 64 22.6 and 12.8; 2 of 20001 and 50001 with 8 of 8, 555 work-groups of 256 tokens: 36.3 and 39.4)
+    // Shorter tiles where those leave compute units idle, until there are two work-groups for each (256 and 64 tokens, calls of one
+    // kind back to back: one sequence of 4000 tokens with 8 kv heads of 4 query heads 10.7 and 4.8 us, 8 of 500..2000 with the same
+    // heads 13.4 and 6.4, 24 of 128..3001 with heads of 64 21.7 and 11.8 (15.4 among the other kernels of a decode step); 2 of 20001 and
+    // 50001 with 8 of 8, 555 work-groups of 256 tokens: 36.3 and 39.4)
     const int64_t wantedGroups = 2 * static_cast<int64_t>(deviceInfo().numCU);
     const int64_t tokens = tokensAtMost(a);
     while (TT > shortest && gridX * ceilDiv(tokens, TT) < wantedGroups) TT /= 2;
@@ -334,9 +335,9 @@ diopiError_t launchStaged(hipStream_t stream, void* out, const void* q, const vo
     // compete with the logits being written (128 sequences of 1024..8192 tokens, 8 kv heads of 8 query heads: 234.3 us against
     // 242.9 with 16 and 243.6 with 8; with one query head per kv head 4 and 8 are 1 % slower than 16), unless work-groups are too
     // few to compete with anything and what counts is how long one takes: then as many as give each of the waves that take the tokens
-    // of a piece in turn a unit of a tile of 64 (one wave, four or more pieces: the first two shapes above 6.6 -> 4.8 and 7.6 -> 6.7 us;
-    // two waves, 2 kv heads of 8 query heads: one sequence of 64 tokens 3.79 us with 16 loads a lane and 3.28 with 8, of 4000 4.09 and
-    // 3.69, and 0.5 more than with 16 with 4; four waves, one kv head of 8: 64 tokens 4.3 with 16 and 3.6 with 4)
+    // of a piece in turn a unit of a tile of 64 (one wave, four or more pieces: the first two shapes above 4.8 -> 4.4 and 6.4 -> 5.8 us;
+    // two waves, 2 kv heads of 8 query heads: one sequence of 64 tokens 3.8 us with 16 loads a lane, 3.2 with 8, 3.4 with 4, of 4000
+    // 4.1, 3.6 and 3.8; four waves, one kv head of 8: 64 tokens 4.3 with 16 and 3.0 with 4)
     if (a.G > 1 && fewGroups && HS == 2) {
         hipLaunchKernelGGL((tokenAttStaged<T, HD, HW, 32>), grid, dim3(kAttThreads), outLds, stream, static_cast<T*>(out), static_cast<const T*>(q),
                            static_cast<const T*>(k), a, TT, HS, scale, order);
