@@ -1079,7 +1079,7 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnPipe(T* 
 // beside it.  Against the pipelined kernel above the balance is the other way round: what pays is more waves a SIMD, which
 // fill each other's waits without a hand-made schedule, so the registers are kept to 3 waves a SIMD: no
 // reference tuple (the multiply-add that scales a score subtracts the reference too) and 64 accumulator registers instead of 96.
-// 8 sequences of 100..2560 tokens, 32 query heads on 8 kv heads, bf16, full attention: 255 us (about 1830 clocks a wave and tile, of
+// 8 sequences of 100..2560 tokens, 32 query heads on 8 kv heads, bf16, full attention: 258 us (about 1850 clocks a wave and tile, of
 // which issuing the vector instructions takes 1620), 4 waves a SIMD the same, work-groups of 8 waves 3 % more, the products dealt
 // out between the next group's exponentials the same; the one-wave-per-row kernel, which heads of 64 took before, 69.5 ms.
 // Layouts as in ctxAttnMfma: S^T and O^T, a lane owns query row lane % 32.  A tile row is 128 bytes, so two rows share the 16
@@ -1128,9 +1128,10 @@ struct Special {
         return static_cast<T>((bits & 0x8000u) ? 128.f : 1.f);
     }
     static __device__ __forceinline__ float value(float count) {  // what the counted ones sum to, 0 if there are none
+        if (!(count < 16384.f)) return __builtin_nanf("");  // may be too large for a whole number
         const int c = static_cast<int>(count);
-        const bool plus = (c & 127) != 0, minus = (c & 16383) >= 128;
-        if (c >= 16384 || (plus && minus)) return __builtin_nanf("");
+        const bool plus = (c & 127) != 0, minus = c >= 128;
+        if (plus && minus) return __builtin_nanf("");
         return plus ? INFINITY : (minus ? -INFINITY : 0.f);
     }
 };
