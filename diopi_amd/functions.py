@@ -68,7 +68,7 @@ def _call(name: str, ctx: Optional[rt.Context], tensor: torch.Tensor, *args):
         ret = op(None, *args)
     else:
         with _on_stream(ctx, tensor):
-            ret = op(ctx.handle.value, *args)
+            ret = op(ctx.handle.value if ctx.handle else 0, *args)  # 0: a closed context, which the operator refuses
     value = None
     if type(ret) is tuple:  # the operators that answer more than their return code
         ret, value = ret

@@ -34,6 +34,13 @@ def test_arguments_that_are_no_tensors_of_a_known_type():
         F.destindex_copy_kv(torch.ones([1] * 9), torch.zeros(1, dtype=torch.int32), torch.ones([1] * 9))
 
 
+def test_a_closed_context_is_refused():
+    ctx = rt.Context(own_stream=True)
+    ctx.close()
+    with pytest.raises(rt.DiopiException):
+        F.rms_norm(torch.ones(2, 4), (4,), torch.ones(4), None, 1e-6, ctx=ctx)
+
+
 def test_a_build_of_the_c_libraries_alone(tmp_path):
     for path in (rt.RT_LIB_PATH, rt.IMPL_LIB_PATH):
         os.symlink(path, tmp_path / os.path.basename(path))
