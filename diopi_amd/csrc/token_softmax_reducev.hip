@@ -82,10 +82,11 @@ __device__ __forceinline__ float waveSumUniform(float v) {
 }
 
 // The last step of a softmax whose logits were all -inf has nothing to divide by: 0 / 0 for heads of 128 as in the reference's
-// softmax, zero for heads of 64 like the general kernel, which served them before.
+// softmax; for heads of 64 what the general kernel gives, which served them before: the sum itself, zero or, with an infinite value or
+// a NaN among the rows, NaN.
 template <int HD>
 __device__ __forceinline__ float weightedSum(float num, float den) {
-    return (HD < kD && den == 0.f) ? 0.f : num / den;
+    return (HD < kD && den == 0.f) ? num : num / den;
 }
 
 // Which (sequence, range) is this work-group's?  The one whose token count has the rank of the work-group's index

@@ -91,6 +91,21 @@ def test_softmax_reducev_infinite_values():
     assert torch.equal(out.isinf(), general.isinf()) and int(out.isinf().sum()) == 8 and not out.isnan().any()
 
 
+@pytest.mark.parametrize("n", [100, 3000])
+def test_softmax_reducev_infinite_values_that_nothing_weighs(n):
+    """A head whose logits are all -inf over rows with an infinite value and a NaN: zeros, and NaN where those stand."""
+    w = _decode([n], 4, 2, torch.float16, torch.int32, 4)
+    w["logits"][1] = -float("inf")
+    w["v"][int(w["b_loc"][0, -1]), 0, 7] = float("inf")
+    w["v"][int(w["b_loc"][0, -n]), 0, 9] = float("nan")
+    out, general = (torch.zeros(1, 4, 64, dtype=torch.float16, device=DEV) for _ in range(2))
+    rest = (w["b_loc"], w["b_start"], w["b_len"], w["longest"], 0)
+    F.token_softmax_reducev(w["logits"], w["v"], out, *rest)
+    F.token_softmax_reducev(w["logits"], _unaligned(w["v"]), general, *rest)
+    assert out[0, 1].isnan().nonzero().flatten().tolist() == [7, 9] and int((out[0, 1] == 0).sum()) == 62
+    assert torch.equal(out[0, 1].isnan(), general[0, 1].isnan())
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("H,Hkv,idt", [(1, 1, torch.int32), (9, 3, torch.int64), (32, 8, torch.int32), (27, 3, torch.int32), (16, 1, torch.int32)])
 def test_token_attention(dt, H, Hkv, idt):
