@@ -1117,7 +1117,8 @@ struct SplitPair<bf16_t> {
 // Infinities and NaN among the values.  A probability of zero keeps nothing out of a product with one (a masked key's, or the lower
 // half of a probability that has none), so a work-group that ends with a NaN anywhere does its tiles again with care: each
 // class is counted among the keys a row sees (1, 2^7 and 2^14 apiece, at most 64 keys: exact in a product) while the product
-// itself takes zeros in their place.
+// itself takes zeros in their place.  However little a key in sight weighs, in exact arithmetic it is more than nothing: a special
+// value counts where its probability has run out, too, and stays when a move of the reference leaves nothing of what was before.
 template <typename T>
 struct Special {
     static constexpr uint32_t kExponent = std::is_same<T, half_t>::value ? 0x7c00u : 0x7f80u;
@@ -1128,7 +1129,7 @@ struct Special {
         return static_cast<T>((bits & 0x8000u) ? 128.f : 1.f);
     }
     static __device__ __forceinline__ float value(float count) {  // what the counted ones sum to, 0 if there are none
-        if (!(count < 16384.f)) return __builtin_nanf("");  // may be too large for a whole number
+        if (count >= 16384.f) return __builtin_nanf("");
         const int c = static_cast<int>(count);
         const bool plus = (c & 127) != 0, minus = c >= 128;
         if (plus && minus) return __builtin_nanf("");
@@ -1318,21 +1319,19 @@ __global__ __launch_bounds__(kWaves64* kWave, 3) void ctxAttn64(T* __restrict__ 
 #pragma unroll
                 for (int mb = 0; mb < D / 32; ++mb) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) o[mb][r] *= alpha;
+                    for (int r = 0; r < 16; ++r) o[mb][r] = (CAREFUL && !__builtin_isfinite(o[mb][r])) ? o[mb][r] : o[mb][r] * alpha;
                 }
             }
         }
         // k slot (hh, j) of group g = 2*sb + u is key 16*g + 8*(j/4) + 4*hh + j%4
         float psum[4] = {0.f, 0.f, 0.f, 0.f};
-        auto probabilities = [&](int g, Frag& hi, Frag& lo, bool (&none)[8]) {
+        auto probabilities = [&](int g, Frag& hi, Frag& lo) {
             FragBits<Frag> h, l;
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[g / 2][8 * (g % 2) + 2 * w], scaleLog2, negRef));
                 const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[g / 2][8 * (g % 2) + 2 * w + 1], scaleLog2, negRef));
                 psum[w] += p0 + p1;
-                none[2 * w] = p0 == 0.f;
-                none[2 * w + 1] = p1 == 0.f;
                 uint32_t hw, lw;
                 Split::split(p0, p1, hw, lw);
                 h.raw[w] = hw;
@@ -1352,13 +1351,10 @@ __global__ __launch_bounds__(kWaves64* kWave, 3) void ctxAttn64(T* __restrict__ 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             Frag hi, lo, seen;
-            bool none[8];
-            probabilities(g, hi, lo, none);
+            probabilities(g, hi, lo);
             if constexpr (CAREFUL) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {  // a key in sight whose probability has run out makes a NaN of whatever is special in its row
-                    seen[j] = static_cast<T>(key0 + 16 * g + 8 * (j / 4) + 4 * hh + j % 4 <= lastKey ? (none[j] ? 16384.f : 1.f) : 0.f);
-                }
+                for (int j = 0; j < 8; ++j) seen[j] = static_cast<T>(key0 + 16 * g + 8 * (j / 4) + 4 * hh + j % 4 <= lastKey ? 1.f : 0.f);
             }
 #pragma unroll
             for (int mb = 0; mb < D / 32; ++mb) {

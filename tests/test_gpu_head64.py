@@ -259,6 +259,26 @@ def test_attention_values_that_are_no_numbers(dt):
     assert ((out - general).abs()[fine].float() <= 3 * ROUND[dt][0] * general.abs()[fine].float() + 1e-3).all()
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("late", [False, True])
+def test_attention_infinite_values_of_keys_that_weigh_little(dt, late):
+    """2^-135 of another key's weight, below the normal numbers of fp32, is still something: infinite values stay infinite, whichever key
+    comes first."""
+    n = 200
+    q, k = torch.zeros(n, 1, 64), torch.zeros(n, 1, 64)
+    q[:, 0, 0] = 8
+    light, heavy = (3, 150) if late else (150, 3)
+    k[heavy, 0, 0] = 135 * np.log(2)
+    v = torch.randn(n, 1, 64, generator=torch.Generator().manual_seed(12))
+    v[light, 0, 5], v[light, 0, 6], v[heavy, 0, 9], v[light + 1, 0, 9] = float("inf"), -float("inf"), float("inf"), -float("inf")
+    q, k, v = (t.to(dt).to(DEV) for t in (q, k, v))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    out = F.flash_attention_varlen(q, k, v, cu, cu, None, n, n, 0.0, None, False)[:, 0]
+    assert out[:, 5].isposinf().all() and out[:, 6].isneginf().all() and out[:, 9].isnan().all()
+    rest = [d for d in range(64) if d not in (5, 6, 9)]
+    assert torch.equal(out[:, rest], v[heavy, 0, rest].expand(n, -1))
+
+
 @pytest.mark.parametrize("scale", [-0.125, 1e-20])
 def test_attention_odd_scales(scale):
     q, k, v, start = _packed([70, 130], 2, 2, torch.float16, 6)
