@@ -71,6 +71,7 @@ struct CtxArgs {
     bool causal;
     int G;             // query heads per key/value head
     float scaleLog2;   // softmax scale * log2(e)
+    double lnPerLog2;  // softmax scale / scaleLog2: ln 2 but for the rounding of scaleLog2 (set for heads of 64)
     float* lse;        // [batch, H, lseStride] log-sum-exp of the scaled scores of every query row, or null
     int lseStride;     // max_seqlen_q
 };
@@ -1086,26 +1087,28 @@ __global__ __launch_bounds__(NWV * kWave, NWV == 4 ? 2 : 1) void ctxAttnPipe(T* 
 // slots of a 256-byte line, and the swizzle is by the row pair:
 //   K tile: slot s of row r holds packet s ^ ((r / 2) & 7)        (16 lanes reading one packet of 16 rows hit 16 slots)
 //   V tile: slot s of row r holds packet s ^ (4 * ((r / 2) & 1))  (the 4 packets of 4 rows that a transposing read takes, too)
-// Both halves are rounded to nearest, so what a split leaves off has no direction.  Where a new reference puts a row's largest
-// probability, and how large one may grow before the reference moves again (powers of two): fp16 runs out of exponents at 2^-24,
-// so its probabilities are kept as large as they can be, 2^11 .. 2^15 for the largest, and what is left off is at most 2^-36 of that one
-// (with the largest at 1 and halves cut toward zero 32768 keys 2^-20 below one other came out 2.5 % short; now within 2^-16).
+// Both halves are rounded to nearest, so what a split leaves off has no direction.  fp16 runs out of exponents at 2^-24, so its
+// probabilities are split at kScale times their size, and the reference moves before one would grow above 2^kMostLog2, to which
+// the largest of a row is 1 at least: 2^11 .. 2^15 after scaling, and what is left off is at most 2^-36 of it (with the largest
+// at 1 and halves cut toward zero 32768 keys 2^-20 below one other came out 2.5 % short; now within 2^-16).  The scale is a
+// multiplication, not a part of the exponent: an exponent of 11 has steps of 2^-20, which a log-sum-exp near zero would show.
 template <typename T>
 struct SplitPair;
 template <>
 struct SplitPair<half_t> {
-    static constexpr float kTopLog2 = 11.f, kMostLog2 = 15.f;
+    static constexpr float kScale = 2048.f, kMostLog2 = 4.f;
     static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& lo) {
         typedef float f32x2 __attribute__((ext_vector_type(2)));
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        const h2 h = __builtin_convertvector((f32x2{a, b}), h2);
+        const float as = a * kScale, bs = b * kScale;
+        const h2 h = __builtin_convertvector((f32x2{as, bs}), h2);
         hi = __builtin_bit_cast(uint32_t, h);
-        lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a - static_cast<float>(h[0]), b - static_cast<float>(h[1])}), h2));
+        lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{as - static_cast<float>(h[0]), bs - static_cast<float>(h[1])}), h2));
     }
 };
 template <>
 struct SplitPair<bf16_t> {
-    static constexpr float kTopLog2 = 0.f, kMostLog2 = kLazyLog2;
+    static constexpr float kScale = 1.f, kMostLog2 = kLazyLog2;
     static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& lo) {
         typedef float f32x2 __attribute__((ext_vector_type(2)));
         hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
@@ -1311,7 +1314,7 @@ __global__ __launch_bounds__(kWaves64* kWave, 3) void ctxAttn64(T* __restrict__ 
         using Split = SplitPair<T>;
         const float lag = __builtin_fmaf(tmax, scaleLog2, negRef);
         if (jt == 0 || __any(lag > Split::kMostLog2)) {
-            const float up = jt == 0 ? lag - Split::kTopLog2 : fmaxf(lag - Split::kTopLog2, 0.f);
+            const float up = jt == 0 ? lag : fmaxf(lag, 0.f);
             const float alpha = __builtin_amdgcn_exp2f(-up);
             negRef -= up;
             if (jt > 0) {
@@ -1429,11 +1432,13 @@ __global__ __launch_bounds__(kWaves64* kWave, 3) void ctxAttn64(T* __restrict__ 
 
     // ---- normalise, transpose through LDS, write rows with 16-byte stores ----
     const float lTot = lRun + __shfl_xor(lRun, 32, kWave);
-    const float inv = 1.0f / lTot;
+    const float inv = (1.0f / SplitPair<T>::kScale) / lTot;
+    // The reference goes back to the unit of the scores by the factor that took it to powers of two, the logarithm is taken of the
+    // mantissa alone, and only the sum is rounded.
     if (a.lse != nullptr && hh == 0 && qRow < L && qRow < a.lseStride) {
-        constexpr float kTop = SplitPair<T>::kTopLog2;  // taken out of both terms: neither is larger, or rounds coarser, for it
+        const double log2Sum = __builtin_amdgcn_frexp_expf(lTot) + static_cast<double>(__builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(lTot)));
         a.lse[(static_cast<int64_t>(planned.x) * a.H + head) * a.lseStride + qRow] =
-            0.6931471805599453f * (__builtin_amdgcn_logf(lTot * __builtin_amdgcn_exp2f(-kTop)) + (kTop - negRef));
+            static_cast<float>(log2Sum * 0.6931471805599453 - static_cast<double>(negRef) * a.lnPerLog2);
     }
     waitLdsLoads();
     __syncthreads();  // the tiles are dead and no request is in flight
@@ -1617,11 +1622,13 @@ diopiError_t dispatchAttention(diopiContextHandle_t ctx, hipStream_t stream, con
     const bool fast = (D == kHD || (D == 64 && scales)) && aligned && planFits && tileFits;
     // 256-row query tiles (8 waves share each K/V tile) once the sequences are long enough to fill them
     const bool wide = a.rows >= 1024 * static_cast<int64_t>(a.batch);
+    CtxArgs a64 = a;
+    a64.lnPerLog2 = softmaxScale / static_cast<double>(a.scaleLog2);
     bool unplanned = false;
     switch (vQ.dtype) {
         case diopi_dtype_float16:
             if (fast && D == 64) {
-                ROCM_CALL((launchMfma<half_t, 4, GEN, 64>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a, store, &unplanned)));
+                ROCM_CALL((launchMfma<half_t, 4, GEN, 64>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a64, store, &unplanned)));
                 if (!unplanned) return diopiSuccess;
             }
             return fast && D == kHD ? (wide ? launchMfma<half_t, 8, GEN, kHD>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a, store)
@@ -1629,7 +1636,7 @@ diopiError_t dispatchAttention(diopiContextHandle_t ctx, hipStream_t stream, con
                         : launchGeneric<half_t, float>(stream, vOut.data, vQ.data, vK.data, vV.data, a, D, softmaxScale);
         case diopi_dtype_bfloat16:
             if (fast && D == 64) {
-                ROCM_CALL((launchMfma<bf16_t, 4, GEN, 64>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a, store, &unplanned)));
+                ROCM_CALL((launchMfma<bf16_t, 4, GEN, 64>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a64, store, &unplanned)));
                 if (!unplanned) return diopiSuccess;
             }
             return fast && D == kHD ? (wide ? launchMfma<bf16_t, 8, GEN, kHD>(ctx, stream, vOut.data, vQ.data, vK.data, vV.data, a, store)

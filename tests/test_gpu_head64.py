@@ -260,6 +260,26 @@ def test_attention_values_that_are_no_numbers(dt):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_attention_log_sum_exp_near_zero(dt, n):
+    """Rows of a few keys with small scores, which are exact in fp32: the log-sum-exp keeps the relative precision of its terms."""
+    B = 200
+    g = torch.Generator().manual_seed(n)
+    q, k = torch.zeros(B * n, 1, 64), torch.zeros(B * n, 1, 64)
+    q[:, 0, 0] = 8
+    k[:, 0, 0] = torch.randn(B * n, generator=g) * 0.05
+    q, k = (t.to(dt).to(DEV) for t in (q, k))
+    cu = torch.arange(B + 1, dtype=torch.int32, device=DEV) * n
+    F.flash_attention_varlen(q, k, k, cu, cu, None, n, n, 0.0, None, False)
+    lse = F.GLOBAL_STATE["flash_attention_varlen_softmax_lse"][:, 0].double()
+    s = k[:, 0, 0].double().view(B, n)
+    want = s.logsumexp(1, keepdim=True)
+    # the reference rounded, and the result; with more than one key their exponents, exponentials, sum and logarithm
+    bound = 2.02 * 2.0 ** -24 * (s.abs().amax(1, keepdim=True) + want.abs()) + (6 * 2.0 ** -24 if n > 1 else 0)
+    assert ((lse - want).abs() <= bound).all(), float(((lse - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("late", [False, True])
 def test_attention_infinite_values_of_keys_that_weigh_little(dt, late):
     """2^-135 of another key's weight, below the normal numbers of fp32, is still something: infinite values stay infinite, whichever key
